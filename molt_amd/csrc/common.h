@@ -15,6 +15,20 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 #define MOLT_DEV __device__ __forceinline__
 
 // ---------------------------------------------------------------------------
+// Vector-memory order. A partial vmcnt wait names operations by their place in
+// issue order: "at most N outstanding" means the N youngest. The compiler knows
+// which registers a load fills, but not that LDS filled by DMA is read after a
+// wait written by hand, so it may issue the operations that such a wait leaves
+// in flight ahead of the ones it waits for (it did: two DMA blocks then landed
+// after the barrier, and other waves read stale LDS rows). Call this between
+// the two groups: what comes before it is issued before what comes after.
+// ---------------------------------------------------------------------------
+MOLT_DEV void loads_in_order() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// ---------------------------------------------------------------------------
 // bf16 conversion. fp32 -> bf16 is round-to-nearest-even (v_cvt_pk_bf16_f32),
 // the same rounding torch applies in `.to(torch.bfloat16)`.
 // ---------------------------------------------------------------------------

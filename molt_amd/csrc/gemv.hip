@@ -940,6 +940,7 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
       for (int b = 0; b < GL_BW; ++b) gl_load_x<1>(xr, xs + 1024 * b, p, blk + min(b, nb - 1), lane);
       __builtin_amdgcn_sched_barrier(0);
       gl_load(b0, s0, p, wr, grp(0), blk, nb, lane, jc);
+      loads_in_order();                      // round 0's wait counts every load of round 1 as younger
       if constexpr (!ONE) gl_load(b1, s1, p, wr, grp(1), blk, nb, lane, jc);
       __builtin_amdgcn_sched_barrier(0);
       gl_wait_vm<(ONE ? 1 : 2) * GlRound<SM, LV>::kLoads>();

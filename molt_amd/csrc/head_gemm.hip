@@ -117,6 +117,7 @@ __global__ __launch_bounds__(NT) void head_grad_kernel(const HeadGradParams p) {
     // sub-step's MFMAs run under the next step's first reads.
     w_load(wb0, 0);
     d_load(db0, 0);
+    loads_in_order();
     w_load(wb1, 1);
     wait_vm_at_most<kStageDma>();
     step_barrier();
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(NT) void head_grad_kernel(const HeadGradParams p) {
       load_frags_nn(wc, dc, ao, bo, 0, a[0], bf[0]);
       mfma_set(a[1], bf[1], acc);
       d_load(dnx, j + 1);
-      dma_then_loads();
+      loads_in_order();
       w_load(w2, j + 2);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll

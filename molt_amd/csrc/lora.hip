@@ -406,6 +406,7 @@ __global__ __launch_bounds__(64 * PJ_WAVES) void lora_project_dma_kernel(const P
     uint16_t* z2 = zs2[NB == 3 ? wave : 0];
     dma(s, z0);
     pj_load_w<TQ>(w0, wr, s, lane);
+    loads_in_order();
     if constexpr (NB == 3) dma(clamp(s + PJ_WAVES), z1);
     // step with z(s) in zc and the adapter in wc; zn receives the z load it issues
     auto step = [&](const u32x4_t (&wc)[TQ][4], u32x4_t (&wn)[TQ][4], const uint16_t* zc, uint16_t* zn) {
@@ -770,6 +771,7 @@ MOLT_DEV void grad_dma_tile(const GradParams& p, int bx, int by, int bz) {
   f32x16_t acc[2][1];
   zero_acc(acc);
   dma(0, la, ra);
+  loads_in_order();
   dma(1, lb, rb);
   pj_wait_vm<3>();                   // stage 0 landed; stage 1 may fly
   pj_barrier();

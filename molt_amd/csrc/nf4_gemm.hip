@@ -850,7 +850,7 @@ MOLT_DEV void wt_tile_write(const FwdParams& p, const uint16_t* __restrict__ wc,
 
 // One thread's packed W bytes and block scale for one forward step. w_load
 // fetches them with exactly kLoads vector-memory instructions, issued after the
-// step's X DMA (dma_then_loads); the step's closing wait leaves exactly these in
+// step's X DMA (loads_in_order); the step's closing wait leaves exactly these in
 // flight, so kLoads is also that wait's vmcnt.
 struct WBytes {
   u32x4_t q;
@@ -1173,6 +1173,7 @@ __global__ __launch_bounds__(NT) void fwd_kernel(const FwdParams p) {
     // step ahead (its tiles are shared by every row block, mostly from L2).
     x_src(xb0, 0);
     w_src(wb0, 0);
+    loads_in_order();
     x_src(xb1, 1);
     wait_vm_at_most<kStageDma>();                    // X(0), W(0) landed; X(1) may fly
     step_barrier();
@@ -1194,7 +1195,7 @@ __global__ __launch_bounds__(NT) void fwd_kernel(const FwdParams p) {
       load_frags(wc, xc, fo, 0, a[0], b[0]);
       mfma_set(a[1], b[1], acc);
       w_src(wnx, j + 1);
-      dma_then_loads();                              // keep W(j + 1) issued before X(j + 2)
+      loads_in_order();                              // keep W(j + 1) issued before X(j + 2)
       x_src(x2, j + 2);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1231,7 +1232,7 @@ __global__ __launch_bounds__(NT) void fwd_kernel(const FwdParams p) {
       load_frags(wc, xc, fo, 0, a[0], b[0]);
       mfma_set(a[1], b[1], acc);
       x_load(xn, k1);
-      dma_then_loads();
+      loads_in_order();
       w_load(nw, k2);
       w_lookup(cw, tabc, 0, c);
       __builtin_amdgcn_sched_barrier(0);
@@ -1659,6 +1660,7 @@ __global__ __launch_bounds__(NT) void bwd_kernel(const BwdParams p) {
     // step ahead (as in the staged forward kernel).
     x_load(xb0, sbeg);
     w_dma(wb0, sbeg);
+    loads_in_order();
     x_load(xb1, sbeg + 1);
     wait_vm_at_most<kStageDma>();                    // dY(sbeg), W(sbeg) landed; dY(sbeg + 1) may fly
     step_barrier();
@@ -1666,7 +1668,7 @@ __global__ __launch_bounds__(NT) void bwd_kernel(const BwdParams p) {
       load_frags(wc, xc, fo, 0, a[0], b[0]);
       mfma_set(a[1], b[1], acc);
       w_dma(wnx, s + 1);
-      dma_then_loads();                              // keep W(s + 1) issued before dY(s + 2)
+      loads_in_order();                              // keep W(s + 1) issued before dY(s + 2)
       x_load(x2, s + 2);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1720,7 +1722,7 @@ __global__ __launch_bounds__(NT) void bwd_kernel(const BwdParams p) {
       load_frags(wc, xc, fo, 0, a[0], b[0]);
       mfma_set(a[1], b[1], acc);
       x_load(xn, s + 1);
-      dma_then_loads();
+      loads_in_order();
       w_load(nw, s + 2);
       wp_lookup(cw, tabc, 0, c);
       __builtin_amdgcn_sched_barrier(0);
@@ -2034,7 +2036,6 @@ namespace mid {
 
 using big::buf_load_lds16;
 using big::dma_slot;
-using big::dma_then_loads;
 using big::FragOff;
 using big::loff;
 using big::make_rsrc;
@@ -2118,8 +2119,11 @@ MOLT_DEV void contract(const Operands& o, int sbeg, int send, bool lora, const i
 #pragma unroll
   for (int j = 0; j < TN; ++j) b[1][j] = bf16x8_t{};
   load(x0, w0, 0);
+  loads_in_order();
   load(x1, w1, 1);
+  loads_in_order();
   load(x2, w2, 2);
+  loads_in_order();
   load(x3, w3, 3);
   wait_vm<3 * kDma>();                               // step 0 landed
   step_barrier();

@@ -98,17 +98,6 @@ MOLT_DEV void wait_vm_at_most() {
 }
 MOLT_DEV void wait_vm0() { wait_vm_at_most<0>(); }
 
-// The end of a step waits with a partial vmcnt that counts the register loads
-// of the next-but-one step as the only ones allowed to stay in flight; that
-// holds only if every DMA of the step is issued before them. vmcnt counts in
-// issue order, so the scheduler must not move a register load above a DMA
-// (it did: two X DMA blocks then landed after the barrier, and other waves
-// read stale LDS rows). Compiler and scheduling barrier between the two groups.
-MOLT_DEV void dma_then_loads() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
 // Workgroup barrier without __syncthreads()'s release fence: the fence makes
 // the compiler drain every outstanding vector-memory op, including register
 // loads of packed weight bytes that are only used a step later. The caller
