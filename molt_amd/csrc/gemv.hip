@@ -672,22 +672,24 @@ void nf4_gemv_dot_kernel(const GemvParams p, int rounds) {
 //   M = 5    7.06 6.57 6.78  13.96 13.75 14.04  17.44 16.49 16.85  10.52 7.93 7.62   14.00 10.64 10.40  7.38 6.70 6.04
 //   M = 8    7.79 7.13 6.82  14.33 14.28 14.31  18.28 17.28 17.03  11.16 8.34 7.72   15.24 11.18 10.53  7.79 7.35 6.07
 //   M = 16   9.11 8.46 7.44  16.13 15.53 15.06  19.90 18.48 17.91  12.64 9.44 8.32   18.04 12.21 11.04  9.01 8.64 6.50
+// Ranks that are no multiple of 8 take B by the same two loads a round; one load and address per rank cost, M = 5:
+// 14336 x 4096 at rank 4 / 5 / 12 21.8 / 21.2 / 22.2 -> 14.2 / 15.4 / 13.8, 8960 x 1600 16.9 / 16.0 / 17.6 -> 9.9 /
+// 10.4 / 9.7 (weights through registers, ranks by fours: 14.2 / 16.1 / 13.7, 10.7 / 10.7 / 10.9).
 constexpr int GL_WAVES = 16, GL_NT = 64 * GL_WAVES, GL_BW = 4;     // GL_BW: blocks of a wave
 constexpr int GL_SLOT = 16 * GL_BW * 32;                 // bytes of one wave's slot
 constexpr int GL_ROT = 1;                                // row >> GL_ROT: see gl_pos
 
 // mode 0: resolved fp32 scales; 1: nested (dq_block >= 4), one u8 code per
 // block; 2: nested, the codes of 4 blocks in one 4-byte load sharing one absmax2
-// entry. LV: 0 no LoRA; 1 T and LoRA B rows read as 16-byte vectors
-// (r % 8 == 0, 16-byte aligned); 2 one value at a time.
+// entry. LV: 0 no LoRA; 1 whole groups of four ranks (r % 4 == 0, T
+// rows 8-byte aligned); 2 any rank.
 template <int SM, int LV>
 struct GlRound {
   static constexpr int NS = SM == 2 ? 1 : SM == 1 ? 2 : GL_BW, NQ = SM == 0 ? 0 : SM == 2 ? 1 : GL_BW;
-  static constexpr int NL = LV == 0 ? 0 : LV == 1 ? 2 : 8;
+  static constexpr int NL = LV == 0 ? 0 : 2;
   static constexpr int kLoads = GL_SLOT / 1024 + NS + NQ + NL;   // vector-memory operations of a round
   uint32_t q[SM == 0 ? 1 : NQ];
   float s[NS];
-  int first;                                               // mode 1: blocks of entry s[0]; the others are s[1]'s
   float lb[8];
 };
 
@@ -716,9 +718,20 @@ MOLT_DEV uint32_t gl_mul(int n, int k) {
   return v;
 }
 
+// Ranks that are no groups of four: byte offset in B of half h of a lane's 8 entries of row n (16 bytes, which need
+// 4-byte alignment only). Kept inside B: a load that straddled its end might lose the entries before it; moved back, it
+// holds them gl_b_shift further up.
+MOLT_DEV uint32_t gl_b_at(const GemvParams& p, int n, int nr, int h) { return (gl_mul(n, p.r) + (uint32_t)(p.r - nr + 4 * h)) * 4u; }
+MOLT_DEV uint32_t gl_b_offset(const GemvParams& p, int n, int nr, int h) {
+  return min(gl_b_at(p, n, nr, h), ((uint32_t)p.N * (uint32_t)p.r - 4u) * 4u);
+}
+MOLT_DEV uint32_t gl_b_shift(const GemvParams& p, int n, int nr, int h) {
+  return (gl_b_at(p, n, nr, h) - gl_b_offset(p, n, nr, h)) / 4u;
+}
+
 template <int SM, int LV>
-MOLT_DEV void gl_load(GlRound<SM, LV>& R, uint8_t* slot, const GemvParams& p, __amdgpu_buffer_rsrc_t wr, int grp, int blk,
-                      int nb, int lane, int jc) {
+MOLT_DEV void gl_load(GlRound<SM, LV>& R, uint8_t* slot, const GemvParams& p, __amdgpu_buffer_rsrc_t wr,
+                      __amdgpu_buffer_rsrc_t br, int grp, int blk, int nb, int lane, int nr) {
   // rows past N repeat the last one and feed only outputs that are not stored;
   // blocks past the slice repeat its last one and are not consumed
 #pragma unroll
@@ -749,21 +762,23 @@ MOLT_DEV void gl_load(GlRound<SM, LV>& R, uint8_t* slot, const GemvParams& p, __
     if constexpr (SM == 1) {                 // 4 blocks lie in at most two groups of dq_block >= 4
       R.s[0] = p.absmax2[(b0 + (uint32_t)min(0, nb - 1)) >> p.dq_shift];
       R.s[1] = p.absmax2[(b0 + (uint32_t)(nb - 1)) >> p.dq_shift];
-      R.first = (1 << p.dq_shift) - (int)(b0 & ((1u << p.dq_shift) - 1));
     }
   }
-  const int j = jc + 8 * (lane >> 4);                                  // first rank of the lane's 8
-  if constexpr (LV == 1) {
+  // The lane's 8 entries of B's row (an address and a load per rank spilled registers, whose reloads waited for the
+  // stream). Ranks past r read what follows and are masked where they are used. Lanes without any read zeros from past
+  // B's end, without traffic, where the offset is not clamped.
+  if constexpr (LV != 0) {
+    const uint32_t row = LV == 1 ? gl_mul(n, p.r) * 4u + (nr > 0 ? (uint32_t)(p.r - nr) * 4u : 0x80000000u) : 0u;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int jj = j + 4 * h;
-      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(p.lb + (int64_t)n * p.r + (jj < p.r ? jj : p.r - 4));
+      const uint32_t off = LV == 1 ? row + 16u * h : gl_b_offset(p, n, nr, h);
+      const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(br, off, 0, 0);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) R.lb[4 * h + e] = v[e];
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t w = v[e];
+        R.lb[4 * h + e] = __builtin_bit_cast(float, w);
+      }
     }
-  } else if constexpr (LV == 2) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) R.lb[e] = p.lb[(int64_t)n * p.r + (j + e < p.r ? j + e : p.r - 1)];
   }
 }
 
@@ -782,8 +797,13 @@ MOLT_DEV void gl_load_x(__amdgpu_buffer_rsrc_t xr, uint8_t* slot, const GemvPara
 
 template <int SM, int LV>
 MOLT_DEV f32x4_t gl_compute(const GlRound<SM, LV>& R, const uint8_t* slot, const GemvParams& p, GlSmem& sm, uint32_t lb,
-                            const u32x4_t (&xf)[GL_BW][2], const u32x4_t& tf, int nb, int nr, int lane) {
+                            const u32x4_t (&xf)[GL_BW][2], const u32x4_t& tf, int grp, int blk, int nb, int nr, int lane) {
   const int col = lane & 15, g = lane >> 4;
+  int first = 0;                       // mode 1: blocks of entry s[0]; the others are s[1]'s
+  if constexpr (SM == 1) {
+    const uint32_t b0 = gl_mul(min(16 * grp + col, (int)p.N - 1), p.K >> 6) + (uint32_t)blk;
+    first = (1 << p.dq_shift) - (int)(b0 & ((1u << p.dq_shift) - 1));
+  }
   u32x2_t w[GL_BW];
 #pragma unroll
   for (int b = 0; b < GL_BW; ++b)
@@ -796,7 +816,7 @@ MOLT_DEV f32x4_t gl_compute(const GlRound<SM, LV>& R, const uint8_t* slot, const
       sc[b] = R.s[b];
     } else {
       const uint32_t q = SM == 2 ? (R.q[0] >> (8 * b)) & 0xffu : R.q[SM == 2 ? 0 : b];
-      const float prod = *gl_code2(sm, q) * (SM == 2 || b < R.first ? R.s[0] : R.s[1]);
+      const float prod = *gl_code2(sm, q) * (SM == 2 || b < first ? R.s[0] : R.s[1]);
       sc[b] = prod + p.offset;
     }
   }
@@ -826,13 +846,26 @@ MOLT_DEV f32x4_t gl_compute(const GlRound<SM, LV>& R, const uint8_t* slot, const
     // be infinite, and zero times that is not zero. Masked when it is used: at
     // its load the select would wait for it.
     u32x4_t bw;
-    if constexpr (LV == 1) {               // ranks of 8: all or none
+    if constexpr (LV == 1) {               // ranks of 4: all or none
 #pragma unroll
-      for (int e = 0; e < 4; ++e) bw[e] = nr > 0 ? pack_bf16x2(p.s * R.lb[2 * e], p.s * R.lb[2 * e + 1]) : 0u;
+      for (int e = 0; e < 4; ++e) bw[e] = nr > 4 * (e >> 1) ? pack_bf16x2(p.s * R.lb[2 * e], p.s * R.lb[2 * e + 1]) : 0u;
     } else {
+      float b[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) b[e] = R.lb[e];
+      if (16 * grp + 15 >= (int)p.N - 4) {   // uniform: the rows whose loads may have been moved back
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const uint32_t sh = gl_b_shift(p, min(16 * grp + col, (int)p.N - 1), nr, h);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) b[4 * h + e] = sh & 1 ? b[4 * h + (e < 3 ? e + 1 : 3)] : b[4 * h + e];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) b[4 * h + e] = sh & 2 ? b[4 * h + e + 2] : b[4 * h + e];
+        }
+      }
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        bw[e] = pack_bf16x2(2 * e < nr ? p.s * R.lb[2 * e] : 0.0f, 2 * e + 1 < nr ? p.s * R.lb[2 * e + 1] : 0.0f);
+        bw[e] = pack_bf16x2(2 * e < nr ? p.s * b[2 * e] : 0.0f, 2 * e + 1 < nr ? p.s * b[2 * e + 1] : 0.0f);
     }
     const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
     const f32x4_t v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8v, tf),
@@ -894,6 +927,7 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
   if constexpr (SM != 0) c2 = p.code2[tid & 255];
   const int mc = col < p.M ? col : p.M - 1;
   u32x4_t tf = {0u, 0u, 0u, 0u};
+  uint32_t tr8[8];                         // LV 2: T's entries as loaded, packed once they have landed
   if constexpr (LV != 0) {
     // Ranks past r, and waves without ranks of this slice, load from outside the
     // buffer: zeros, no traffic (T gathered by all waves cost 0.4 us a token) and
@@ -904,18 +938,22 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
     const uint32_t row = gl_mul(mc, (int)p.ldt) * 2u;
     auto at = [&](int jj) { return lora && jj < p.r ? row + 2u * (uint32_t)jj : 0xfffffff0u; };
     if constexpr (LV == 1) {
-      tf = __builtin_amdgcn_raw_buffer_load_b128(tr, at(j), 0, 0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(tr, at(j + 4 * h), 0, 0);
+        tf[2 * h] = v[0]; tf[2 * h + 1] = v[1];
+      }
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        tf[i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(tr, at(j + 2 * i), 0, 0) |
-                ((uint32_t)__builtin_amdgcn_raw_buffer_load_b16(tr, at(j + 2 * i + 1), 0, 0) << 16);
+      for (int i = 0; i < 8; ++i) tr8[i] = __builtin_amdgcn_raw_buffer_load_b16(tr, at(j + i), 0, 0);
     }
   }
   __builtin_amdgcn_sched_barrier(0);       // the small loads stay ahead of the weight stream
 
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t*>(p.packed), (short)0, (int)(p.N * (p.K >> 1)), 0x00020000);
+  const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(p.lb), (short)0, (int)(p.N * p.r * 4), 0x00020000);
   // group of round j: rounds past the last repeat the workgroup's own last one (never computed)
   const int glast = (int)((p.N - 1) >> 4), per = (int)gridDim.x * gpr;
   auto grp = [&](int j) { return min(min(j, rounds - 1) * per + (int)blockIdx.x * gpr + q, glast); };
@@ -930,6 +968,10 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
   // place. Up to 8 rows all four fit there, and round 1 need not wait for them.
   uint8_t* xs = reinterpret_cast<uint8_t*>(sm.tab) + wave * 2 * GL_SLOT;
   const bool x8 = p.M <= 8;
+  auto pack_t = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) tf[i] = tr8[2 * i] | (tr8[2 * i + 1] << 16);
+  };
   u32x4_t xf[GL_BW][2];
   if (active) {
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
@@ -939,11 +981,12 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
 #pragma unroll
       for (int b = 0; b < GL_BW; ++b) gl_load_x<1>(xr, xs + 1024 * b, p, blk + min(b, nb - 1), lane);
       __builtin_amdgcn_sched_barrier(0);
-      gl_load(b0, s0, p, wr, grp(0), blk, nb, lane, jc);
+      gl_load(b0, s0, p, wr, br, grp(0), blk, nb, lane, nr);
       loads_in_order();                      // round 0's wait counts every load of round 1 as younger
-      if constexpr (!ONE) gl_load(b1, s1, p, wr, grp(1), blk, nb, lane, jc);
+      if constexpr (!ONE) gl_load(b1, s1, p, wr, br, grp(1), blk, nb, lane, nr);
       __builtin_amdgcn_sched_barrier(0);
       gl_wait_vm<(ONE ? 1 : 2) * GlRound<SM, LV>::kLoads>();
+      if constexpr (LV == 2) pack_t();
       asm volatile("" ::"v"(c2), "v"(tf) : "memory");      // older loads, landed: said here, where they can still be counted
 #pragma unroll
       for (int b = 0; b < GL_BW; ++b)
@@ -956,9 +999,10 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
       gl_load_x<2>(xr, xs, p, blk + min(2, nb - 1), lane);
       gl_load_x<2>(xr, xs + GL_SLOT, p, blk + min(3, nb - 1), lane);
       __builtin_amdgcn_sched_barrier(0);
-      gl_load(b0, s0, p, wr, grp(0), blk, nb, lane, jc);
+      gl_load(b0, s0, p, wr, br, grp(0), blk, nb, lane, nr);
       __builtin_amdgcn_sched_barrier(0);
       gl_wait_vm<GlRound<SM, LV>::kLoads>();
+      if constexpr (LV == 2) pack_t();
       asm volatile("" ::"v"(c2), "v"(tf) : "memory");
       const uint8_t* at[GL_BW] = {s1, s2, xs, xs + GL_SLOT};
 #pragma unroll
@@ -968,7 +1012,7 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
       if constexpr (!ONE) {
         __builtin_amdgcn_s_waitcnt(0xC07F);    // the slot of round 1 has been read
         asm volatile("" ::: "memory");
-        gl_load(b1, s1, p, wr, grp(1), blk, nb, lane, jc);
+        gl_load(b1, s1, p, wr, br, grp(1), blk, nb, lane, nr);
       }
     }
   } else {
@@ -1036,11 +1080,11 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
     return;
   }
   auto round = [&](int j, GlRound<SM, LV>& cur, const uint8_t* slot, GlRound<SM, LV>& nxt, uint8_t* into) {
-    if constexpr (!ONE) gl_load(nxt, into, p, wr, grp(j + 2), blk, nb, lane, jc);
+    if constexpr (!ONE) gl_load(nxt, into, p, wr, br, grp(j + 2), blk, nb, lane, nr);
     __builtin_amdgcn_sched_barrier(0);
     gl_wait_vm<kFly>();
     asm volatile("" ::: "memory");
-    const f32x4_t acc = gl_compute(cur, slot, p, sm, lb, xf, tf, nb, nr, lane);
+    const f32x4_t acc = gl_compute(cur, slot, p, sm, lb, xf, tf, grp(j), blk, nb, nr, lane);
     reduce(j, &acc);
   };
   for (int j = 0;;) {
@@ -1310,15 +1354,15 @@ extern "C" int molt_nf4_gemv(const uint16_t* x, int64_t ldx, int64_t M, const mo
   // slower one at every size measured (see nf4_gemv_lds_kernel).
   MOLT_REQUIRE(gl_ws || !gemv_needs_workspace(M, w->cols), MOLT_EWORKSPACE,
                "%s: workspace of %zu bytes (16-byte aligned) needed, got %zu", who, gl_need, workspace_bytes);
-  if (gl_ws && r <= 32 * gl.wpg && M * ldt < (1ll << 30) && aligned(w->packed, 16) && (!nested || w->dq_block >= 4)) {
+  if (gl_ws && r <= 32 * gl.wpg && M * ldt < (1ll << 30) && w->rows * r < (1ll << 29) && (r == 0 || w->rows * r >= 4) && aligned(w->packed, 16) && (!nested || w->dq_block >= 4)) {
     const int64_t sets = ceil_div64(ceil_div64(w->rows, 16), gl.gpr);
     const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(sets, molt::device_cus() / gl.slices));
     const int rounds = (int)ceil_div64(sets, wgs);
     const bool q4u = nested && w->dq_block >= 4 && (w->cols / 64) % 4 == 0 && aligned(w->absmax_q, 4);
     float* part = gl.slices > 1 ? static_cast<float*>(workspace) : nullptr;
     const dim3 grid((unsigned)wgs, (unsigned)gl.slices);
-    // T and LoRA B rows as 16-byte vectors where every 8-rank group is aligned
-    const int lv = r == 0 ? 0 : (r % 8 == 0 && aligned(lora_b, 16) && ldt % 8 == 0 && aligned(t, 16) ? 1 : 2);
+    // whole groups of four ranks: nothing to shift at B's end, T as 8-byte vectors
+    const int lv = r == 0 ? 0 : (r % 4 == 0 && ldt % 4 == 0 && aligned(t, 8) ? 1 : 2);
 #define MOLT_GL(SMv, LVv) \
   do {                                                                                                                  \
     if (rounds == 1)                                                                                                    \

@@ -399,3 +399,29 @@ def test_gemv_infinite_adapter_entry_stays_in_its_row(m, n, k, r):
     assert torch.equal(y[:, 7], sign * float("inf"))
     y[:, 7] = 0.0
     assert torch.isfinite(y).all()
+
+
+@pytest.mark.parametrize("m,n,k,r", [(5, 4133, 4096, 4), (16, 2065, 1600, 12), (9, 4500, 896, 20), (3, 2070, 14336, 36),
+                                     (16, 4100, 1536, 100)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_gemv_streamed_ranks_of_four(m, n, k, r, shift):
+    """Ranks that are a multiple of 4 and not of 8, over one and several rounds and a partial last group: half of the
+    last lanes' ranks exist, the next row's entries (an infinite one among them) follow in memory. ``shift``: B at an
+    address that is not a multiple of 16, which takes its entries one at a time."""
+    print(f"streamed gemv ranks of four m={m} n={n} k={k} r={r} shift={shift}", flush=True)
+    s = 2.0
+    packed, qs = molt_amd.quantize_4bit(seeded((n, k), 600 + k, std=0.02, dtype=torch.float32))
+    x, t = seeded((m, k), 601), seeded((m, r), 602)
+    b = torch.empty(n * r + shift, device="cuda")[shift:].view(n, r)
+    b.copy_(seeded((n, r), 603, std=0.01, dtype=torch.float32))
+    b[11, 0] = b[n - 1, r - 1] = float("inf")
+    y = _gemv(x, packed, qs, t, b, s)
+    assert torch.equal(y, _gemv(x, packed, qs, t, b, s))
+    got, sign = np_f32(y), np.sign(np_f32(t))
+    assert np.array_equal(got[:, 11], sign[:, 0] * np.inf) and np.array_equal(got[:, n - 1], sign[:, r - 1] * np.inf)
+    wo = oracle_weight(packed, qs).dequant_bf16().astype(np.float64)
+    b[11, 0] = b[n - 1, r - 1] = 0.0
+    ref = bf16_values(x) @ wo.T + s * (bf16_values(t) @ bf16_values(b).T)
+    keep = np.ones(n, bool)
+    keep[[11, n - 1]] = False
+    assert_close_fro(got[:, keep], ref[:, keep], what="Y")

@@ -13,6 +13,8 @@ import pytest
 from molt_amd.build import ARCH, LIB
 
 LLVM = "/opt/rocm/llvm/bin/"
+needs_build = pytest.mark.skipif(not (LIB.exists() and shutil.which(LLVM + "llvm-objdump")),
+                                 reason="no built library or no llvm-objdump")
 MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
 
 
@@ -61,7 +63,7 @@ def _memory(instructions: list[str]) -> list[str]:
     return out
 
 
-@pytest.mark.skipif(not (LIB.exists() and shutil.which(LLVM + "llvm-objdump")), reason="no built library or llvm-objdump")
+@needs_build
 def test_streamed_gemv_issues_its_rounds_in_order(tmp_path):
     """Up to 8 tokens, several rounds: the first round's wait leaves the youngest two rounds' loads in flight, so the
     prologue must issue X, all of round 0, then all of round 1: the same pattern of DMA and loads twice."""
@@ -69,7 +71,7 @@ def test_streamed_gemv_issues_its_rounds_in_order(tmp_path):
     assert len(kernels) == 9, sorted(kernels)          # three scale forms by three adapter forms
     for sym, ins in kernels.items():
         sm, lv = (int(v) for v in re.search(r"ILi(\d)ELi(\d)ELb0E", sym).groups())
-        per = 2 + (4, 6, 2)[sm] + (0, 2, 8)[lv]        # two DMAs, statistics, adapter entries
+        per = 2 + (4, 6, 2)[sm] + (0, 2, 2)[lv]        # two DMAs, statistics, adapter entries
         seq = [e for e in _memory(ins) if e in "DL" or e == f"W{2 * per}"]
         heads = ["".join(seq[max(0, i - 4 - 2 * per):i]) for i, e in enumerate(seq) if e not in "DL"]
         heads = [h for h in heads if h.startswith("DDDD") and "W" not in h]
@@ -77,3 +79,22 @@ def test_streamed_gemv_issues_its_rounds_in_order(tmp_path):
         for h in heads:
             rounds = h[4:4 + per], h[4 + per:]
             assert rounds[0].count("D") == rounds[1].count("D") == 2, f"{sym}: {h}"
+        # and each further round issues as many operations as its wait counts (merged loads would not be)
+        between = "".join(e[0] for e in seq).split("W")
+        assert [n for n in map(len, between[-4:-1])] == [per] * 3, f"{sym}: {per} a round, got {between[-4:]}"
+
+
+@needs_build
+def test_streamed_gemv_holds_its_rounds_in_registers(tmp_path):
+    """The streamed GEMV spills no vector registers (a spill's reload waits for the weight stream), but for two in the
+    form of per-block codes and ranks that are no groups of four."""
+    spills = {}
+    for i, code in enumerate(_code_objects()):
+        if b"nf4_gemv_lds_kernel" in code:
+            (tmp_path / f"{i}.co").write_bytes(code)
+            notes = subprocess.run([LLVM + "llvm-readelf", "--notes", str(tmp_path / f"{i}.co")], capture_output=True,
+                                   text=True, check=True).stdout
+            spills.update(re.findall(r"\.name:\s+(\S*nf4_gemv_lds_kernel\S*).*?\.vgpr_spill_count:\s+(\d+)", notes, re.S))
+    assert len(spills) == 18
+    over = {k: int(v) for k, v in spills.items() if int(v) > (2 if "ILi1ELi2ELb0E" in k else 0)}
+    assert not over, over
