@@ -1186,15 +1186,28 @@ using namespace molt;
 namespace molt {
 namespace {
 // Plan of the streaming MFMA kernel: K slices of slice_blocks blocks, waves per
-// group, groups side by side.
+// group, groups side by side. A workgroup holds up to four groups (as many as its
+// waves allow), but only as many as pay: what counts is rounds x groups a round,
+// and among equals the fewer rounds. us, M = 5, as many as fit / as many as pay:
+// 4096 x 896 6.0 / 4.5 (64 workgroups or 256), 2560 x 2048 6.1 / 5.2, 8960 x 896
+// 6.1 / 5.7 (rounds of four or three groups), 8960 x 2048 8.7 / 7.8 (two rounds of
+// two or three of one); 6144 x 1536 5.5 with two groups in one round, 6.5 with one
+// in two.
 struct GlPlan { int slices, slice_blocks, wpg, gpr; };
-GlPlan gl_plan(int64_t K) {
+GlPlan gl_plan(int64_t N, int64_t K) {
   const int KB = (int)(K / 64), most = GL_WAVES * GL_BW;
   const int slices = (KB + most - 1) / most;
   // slices in whole units of GL_BW blocks, as even as they come
   const int sb = (((KB + GL_BW - 1) / GL_BW + slices - 1) / slices) * GL_BW;
   const int wpg = sb / GL_BW;
-  return {(KB + sb - 1) / sb, sb, wpg, std::max(1, std::min(4, GL_WAVES / wpg))};
+  GlPlan g{(KB + sb - 1) / sb, sb, wpg, 1};
+  const int64_t groups = ceil_div64(N, 16), wgs = std::max(1, molt::device_cus() / g.slices);
+  int64_t best = ceil_div64(groups, wgs);
+  for (int n = 2; n <= std::min(4, GL_WAVES / wpg); ++n) {
+    const int64_t cost = n * ceil_div64(ceil_div64(groups, n), wgs);
+    if (cost <= best) { best = cost; g.gpr = n; }
+  }
+  return g;
 }
 // K slices of the fallback MFMA kernel (nf4_gemv_kernel): narrow outputs (at
 // most 128 groups of 16 rows) split K over up to 8 workgroups per group, as
@@ -1221,7 +1234,7 @@ static bool gemv_needs_workspace(int64_t M, int64_t K) {
 extern "C" size_t molt_nf4_gemv_workspace(int64_t M, int64_t N, int64_t K) {
   // fp32 partials of the K slices when the streaming MFMA kernel, or the
   // fallback kernel of a narrow output, splits K
-  const int ks = M >= 2 && K >= 64 ? gl_plan(K).slices : 0;
+  const int ks = M >= 2 && K >= 64 ? gl_plan(N, K).slices : 0;
   const int vs = gv_slices(N, K);
   const int s = std::max(ks, vs);
   return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) : 0;
@@ -1279,7 +1292,7 @@ extern "C" int molt_nf4_gemv(const uint16_t* x, int64_t ldx, int64_t M, const mo
   // two pieces fit in LDS beside the code table): eight tokens per lookup,
   // where the MFMA kernel, with one 16-row group per workgroup, leaves most
   // CUs idle (M = 8: 2048^2 5.4 / 6.8 us, 1536^2 5.3 / 5.6; 1024 x 4096 6.5 / 6.9).
-  const GlPlan gl = gl_plan(w->cols);
+  const GlPlan gl = gl_plan(w->rows, w->cols);
   const size_t gl_need = gl.slices > 1 ? (size_t)gl.slices * (size_t)M * (size_t)w->rows * sizeof(float) : 0;
   const bool gl_ws = gl_need == 0 || (workspace && workspace_bytes >= gl_need && aligned(workspace, 16));
   const int ipr_need = (int)ceil_div64(w->cols, 2048);

@@ -425,3 +425,17 @@ def test_gemv_streamed_ranks_of_four(m, n, k, r, shift):
     keep = np.ones(n, bool)
     keep[[11, n - 1]] = False
     assert_close_fro(got[:, keep], ref[:, keep], what="Y")
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 2560, 512), (9, 4864, 512), (5, 8960, 896), (3, 14336, 512), (16, 4100, 1536),
+                                   (8, 8960, 2048), (12, 40, 896)])
+def test_gemv_streamed_groups_side_by_side(m, n, k):
+    """One to four groups of 16 rows to a workgroup, by the output's width: one (2560 rows, and 8960 at K = 2048), two
+    (4864), three (8960), four (14336), a last round that is partly past the output."""
+    print(f"streamed gemv groups m={m} n={n} k={k}", flush=True)
+    r, s = 16, 2.0
+    packed, qs = molt_amd.quantize_4bit(seeded((n, k), 700 + k, std=0.02, dtype=torch.float32))
+    x, t, b = seeded((m, k), 701), seeded((m, r), 702), seeded((n, r), 703, std=0.01, dtype=torch.float32)
+    y = _gemv(x, packed, qs, t, b, s)
+    wo = oracle_weight(packed, qs).dequant_bf16().astype(np.float64)
+    assert_close_fro(np_f32(y), bf16_values(x) @ wo.T + s * (bf16_values(t) @ bf16_values(b).T), what="Y")
