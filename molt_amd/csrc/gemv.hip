@@ -1231,6 +1231,26 @@ static bool gemv_needs_workspace(int64_t M, int64_t K) {
   return (c % 7 == 0 && c > 7 && c / 7 <= 8) || (c % 7 != 0 && c % 8 == 0 && c / 8 <= 8);
 }
 
+// Kilobyte pieces of a row, and whether the dot kernel serves a call by its
+// sizes (with 16-byte aligned codes). M = 1, 2 always. Up to 8 tokens over at
+// most 2048 rows and K <= 4096 (eight X rows of at most two pieces fit in LDS
+// beside the code table): eight tokens per lookup, where the MFMA kernel leaves
+// most CUs idle (M = 8: 2048^2 5.4 / 6.8 us, 1536^2 5.3 / 5.6; 1024 x 4096 6.5 /
+// 6.9; M = 4: 1536^2 4.0 / 5.3, 2048 x 8192 7.8 / 9.0). M = 3, 4 with three
+// pieces over at most 4096 rows, two rounds of the grid, where the MFMA kernel
+// runs two slices, two or more rounds and their sum (4096 x 4160 8.5 / 11.1 us, 2112
+// x 5120 8.1 / 9.5, 4096 x 6144 8.8 / 11.1; but 4608 x 5120 13.0 / 11.3, and with
+// two or four pieces 4096^2 7.0 / 6.4, 2560 x 7168 11.5 / 10.9). The
+// MOLT_TUNE_GEMV_DOT_M setting (0..8) replaces the rule by a plain bound on M.
+static int64_t dot_pieces(int64_t K) { return ceil_div64(K, 2048); }
+static bool dot_serves(int64_t M, int64_t N, int64_t K) {
+  const int64_t pieces = dot_pieces(K);
+  if (pieces > 7 || (M > 4 && pieces > 2)) return false;
+  const int most = (int)molt::tuning_value(MOLT_TUNE_GEMV_DOT_M);
+  if (most >= 0) return M <= most;
+  return M <= 2 || (M <= 8 && N <= 2048) || (M <= 4 && N <= 4096 && pieces == 3);
+}
+
 extern "C" size_t molt_nf4_gemv_workspace(int64_t M, int64_t N, int64_t K) {
   // fp32 partials of the K slices when the streaming MFMA kernel, or the
   // fallback kernel of a narrow output, splits K
@@ -1280,27 +1300,19 @@ extern "C" int molt_nf4_gemv(const uint16_t* x, int64_t ldx, int64_t M, const mo
   // workgroups as fit on the GPU at once (two per CU at K = 4096 with up to two
   // tokens, else one; at K = 14336 three rounds of 7 KB per wave need ~190
   // registers); the waves loop over the rounds. M = 2 runs with two X rows, 3
-  // and 4 with four. It serves M <= 2, and M = 3, 4 over at most 2048 rows (M = 4,
-  // against the MFMA kernel: 1536^2 4.0 / 5.3 us, 2048 x 8192 7.8 / 9.0, but 4096^2
-  // 7.2 / 6.6, 4096 x 14336 17.6 / 16.6) or without
-  // the workspace for its slices; the MOLT_TUNE_GEMV_DOT_M setting (0..8)
-  // replaces that rule by a plain bound on M.
+  // and 4 with four. It serves the calls of dot_serves, and up to four tokens
+  // without the workspace for the MFMA kernel's slices. Elsewhere that kernel is
+  // the faster one (M = 4: 4096 x 14336 17.6 / 16.6 us).
   // Any K (a multiple of 64, at most 7 pieces of 2048): a row is IPR pieces of
   // 1 KB, the last possibly partial; IPR is rounded up to an instantiated
   // value (a wholly idle piece re-reads the row's last bytes and is dropped).
-  // M = 5..8 over at most 2048 rows and K <= 4096 (eight X rows of at most
-  // two pieces fit in LDS beside the code table): eight tokens per lookup,
-  // where the MFMA kernel, with one 16-row group per workgroup, leaves most
-  // CUs idle (M = 8: 2048^2 5.4 / 6.8 us, 1536^2 5.3 / 5.6; 1024 x 4096 6.5 / 6.9).
   const GlPlan gl = gl_plan(w->rows, w->cols);
   const size_t gl_need = gl.slices > 1 ? (size_t)gl.slices * (size_t)M * (size_t)w->rows * sizeof(float) : 0;
   const bool gl_ws = gl_need == 0 || (workspace && workspace_bytes >= gl_need && aligned(workspace, 16));
-  const int ipr_need = (int)ceil_div64(w->cols, 2048);
-  const int dot_max_m = (int)molt::tuning_value(MOLT_TUNE_GEMV_DOT_M);
-  const bool dot_m = (dot_max_m >= 0 ? M <= dot_max_m
-                                     : (M <= 2 || (M <= 8 && w->rows <= 2048) || (M <= 4 && !gl_ws))) &&
-                     (M <= 4 || ipr_need <= 2);
-  if (dot_m && ipr_need <= 7 && aligned(w->packed, 16)) {
+  const int ipr_need = (int)dot_pieces(w->cols);
+  const bool dot_m = dot_serves(M, w->rows, w->cols) ||
+                     (M <= 4 && ipr_need <= 7 && !gl_ws && molt::tuning_value(MOLT_TUNE_GEMV_DOT_M) < 0);
+  if (dot_m && aligned(w->packed, 16)) {
     const int ipr = ipr_need <= 3 ? ipr_need : (ipr_need <= 5 ? 5 : 7);
     const int cus = molt::device_cus();
     const int rw = 1;                                         // rows per wave per round

@@ -439,3 +439,20 @@ def test_gemv_streamed_groups_side_by_side(m, n, k):
     y = _gemv(x, packed, qs, t, b, s)
     wo = oracle_weight(packed, qs).dequant_bf16().astype(np.float64)
     assert_close_fro(np_f32(y), bf16_values(x) @ wo.T + s * (bf16_values(t) @ bf16_values(b).T), what="Y")
+
+
+@pytest.mark.parametrize("m,n,k,r", [(3, 2112, 4160, 16), (4, 4096, 6144, 24), (3, 4096, 5120, 0), (4, 4097, 4160, 16)])
+def test_gemv_three_and_four_tokens_over_three_pieces(m, n, k, r):
+    """The edges of the dot kernel's rule for three and four tokens: 2112 to 4096 rows of three pieces, partial and
+    whole, and the first width past it."""
+    print(f"gemv three pieces m={m} n={n} k={k} r={r}", flush=True)
+    s = 2.0
+    packed, qs = molt_amd.quantize_4bit(seeded((n, k), 800 + k, std=0.02, dtype=torch.float32))
+    x = seeded((m, k), 801)
+    t = b = None
+    wo = oracle_weight(packed, qs).dequant_bf16().astype(np.float64)
+    ref = bf16_values(x) @ wo.T
+    if r:
+        t, b = seeded((m, r), 802), seeded((n, r), 803, std=0.01, dtype=torch.float32)
+        ref = ref + s * (bf16_values(t) @ bf16_values(b).T)
+    assert_close_fro(np_f32(_gemv(x, packed, qs, t, b, s)), ref, what="Y")
