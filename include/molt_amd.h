@@ -464,7 +464,8 @@ size_t molt_nf4_gemm_backward_workspace(int64_t M, int64_t N, int64_t K, int32_t
  * block_size == 64 and a power-of-two dq_block. molt_nf4_gemv_workspace()
  * returns the workspace size: fp32 partials (slices x M x N) when the kernel
  * for 2 <= M <= 16 splits K over workgroups (one slice per 4096 elements begun;
- * K = 14336: four), else 0. Less is refused where K is 2 to 8 whole slices of
+ * K = 14336: four), else 0 (also where the kernel for few tokens, which does not
+ * split, serves the call). Less is refused where K is 2 to 8 whole slices of
  * 3584 or 4096 elements; elsewhere a slower kernel runs unsplit.
  * Concurrent calls need separate workspaces.
  * Replaces the bnb.matmul_4bit decode path (training/qlora.py:1332-1358). */
@@ -487,16 +488,18 @@ int molt_nf4_lora_gemv(const uint16_t* x, int64_t ldx, int64_t M, const molt_nf4
 /* molt_nf4_gemv without a workspace argument and without any allocation. No
  * counterpart in the reference: it is for callers that cannot allocate (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc). The split-K partials live in a static device array of
- * molt_nf4_gemv_noalloc_limit() bytes (8 MiB) per GPU, held until the process
- * ends; a shape needing more (a workspace that molt_nf4_gemv would not do
- * without, above the limit) returns MOLT_EUNSUPPORTED before any launch. Every call on one GPU shares that GPU's
- * array. Calls from different streams or host threads are ordered: each waits
- * on an event the previous call recorded on its own stream. Calls made during a
- * graph capture are not ordered that way (no wait, no record); replays of such a
- * graph that overlap other calls on the same GPU race. Same results as
- * molt_nf4_gemv given that workspace (none where the query is above the limit),
- * bit for bit. */
+ * hipMalloc). Where K has to be split (the shapes that molt_nf4_gemv refuses less
+ * than its workspace for) or the output is narrow (at most 2048 rows, except
+ * where the kernel for few tokens serves the call), the partials live in a static
+ * device array of molt_nf4_gemv_noalloc_limit() bytes (8 MiB) per GPU, held until
+ * the process ends; a shape that has to split and needs more returns
+ * MOLT_EUNSUPPORTED before any launch. Those calls share that GPU's array. From
+ * different streams or host threads they are ordered: each waits on an event the
+ * previous one recorded on its own stream. Made during a graph capture they are
+ * not ordered that way (no wait, no record); replays of such a graph that overlap
+ * other such calls on the same GPU race. All other calls use no array and share
+ * nothing. Results are those of molt_nf4_gemv, given its workspace by the calls
+ * that use the array and none by the others, bit for bit. */
 size_t molt_nf4_gemv_noalloc_limit(void);
 int molt_nf4_gemv_noalloc(const uint16_t* x, int64_t ldx, int64_t M, const molt_nf4_weight* w,
                           const uint16_t* t, int64_t ldt, const float* lora_b, int32_t r,

@@ -1254,7 +1254,7 @@ static bool dot_serves(int64_t M, int64_t N, int64_t K) {
 extern "C" size_t molt_nf4_gemv_workspace(int64_t M, int64_t N, int64_t K) {
   // fp32 partials of the K slices when the streaming MFMA kernel, or the
   // fallback kernel of a narrow output, splits K
-  const int ks = M >= 2 && K >= 64 ? gl_plan(N, K).slices : 0;
+  const int ks = K >= 64 && (gemv_needs_workspace(M, K) || !dot_serves(M, N, K)) ? gl_plan(N, K).slices : 0;
   const int vs = gv_slices(N, K);
   const int s = std::max(ks, vs);
   return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) : 0;
@@ -1524,6 +1524,17 @@ bool capturing(hipStream_t stream) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
+
+// The calls that take the shared scratch. Everything that shares it is ordered by an event, and captured calls not even
+// that, so a call takes it only where it has to (no kernel serves the shape unsplit) or where a narrow output would
+// leave the GPU idle; elsewhere the dot kernel or the unsplit one-group kernel runs, on any number of streams at once.
+bool noalloc_splits(int64_t M, const molt_nf4_weight* w) {
+  const bool dot = aligned(w->packed, 16) &&
+                   (dot_serves(M, w->rows, w->cols) ||
+                    (M <= 4 && dot_pieces(w->cols) <= 7 && (w->cols == 14336 || !gemv_needs_workspace(M, w->cols)) &&
+                     molt::tuning_value(MOLT_TUNE_GEMV_DOT_M) < 0));
+  return !dot && (gemv_needs_workspace(M, w->cols) || gv_slices(w->rows, w->cols) > 1);
+}
 }  // namespace
 
 extern "C" size_t molt_nf4_gemv_noalloc_limit(void) { return GEMV_SCRATCH_BYTES; }
@@ -1535,13 +1546,12 @@ extern "C" int molt_nf4_gemv_noalloc(const uint16_t* x, int64_t ldx, int64_t M, 
   MOLT_REQUIRE(w != nullptr, MOLT_EINVAL, "%s: null weight", who);
   MOLT_REQUIRE(M >= 1 && M <= 16 && w->rows > 0 && w->cols > 0, MOLT_EUNSUPPORTED, "%s: M=%lld outside 1..16 or empty weight",
                who, (long long)M);
-  size_t need = molt_nf4_gemv_workspace(M, w->rows, w->cols);
-  if (need > GEMV_SCRATCH_BYTES && !gemv_needs_workspace(M, w->cols)) need = 0;   // the kernel that does not split
-  MOLT_REQUIRE(need <= GEMV_SCRATCH_BYTES, MOLT_EUNSUPPORTED,
+  const size_t need = molt_nf4_gemv_workspace(M, w->rows, w->cols);
+  MOLT_REQUIRE(need <= GEMV_SCRATCH_BYTES || !gemv_needs_workspace(M, w->cols), MOLT_EUNSUPPORTED,
                "%s: M=%lld, %lld x %lld needs %zu bytes of split-K partials, more than the %zu-byte static scratch "
                "(use molt_nf4_gemv with a workspace)",
                who, (long long)M, (long long)w->rows, (long long)w->cols, need, GEMV_SCRATCH_BYTES);
-  if (need == 0) return molt_nf4_gemv(x, ldx, M, w, t, ldt, lora_b, r, scaling, y, ldy, nullptr, 0, stream);
+  if (need > GEMV_SCRATCH_BYTES || !noalloc_splits(M, w)) return molt_nf4_gemv(x, ldx, M, w, t, ldt, lora_b, r, scaling, y, ldy, nullptr, 0, stream);
   // Wait, launch and record under one lock, so calls from several host threads
   // are ordered as they take it. Under graph capture the graph's own order
   // applies and the event is neither waited on nor recorded.

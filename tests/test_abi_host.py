@@ -220,6 +220,17 @@ def test_noalloc_gemv_refuses_oversized_partials_before_any_device_call():
     assert b"static scratch" in lib.molt_amd_last_error()
 
 
+def test_gemv_workspace_is_asked_only_where_k_is_split():
+    """The query is zero where the dot kernel serves the call (it has no partials): one and two tokens at any K that
+    needs no slices, three and four over few rows of three pieces. Shapes that refuse less than their workspace, and
+    narrow outputs, which split in the other kernels, keep theirs."""
+    q = _lib.load().molt_nf4_gemv_workspace
+    assert [int(q(*a)) for a in ((2, 4096, 8960), (2, 4096, 5120), (1, 4096, 14336), (3, 4096, 5120), (4, 2112, 4160),
+                                 (16, 4096, 4096))] == [0] * 6
+    assert all(int(q(*a)) > 0 for a in ((2, 4096, 14336), (3, 1024, 14336), (3, 4608, 5120), (5, 4096, 8960),
+                                        (5, 4096, 5120), (16, 1536, 8960)))
+
+
 def test_split_k_workspace_queries_need_no_gpu():
     """The split plan: a long contraction with few 256 x 256 output tiles gets
     fp32 partials for S splits; a problem that fills the GPU gets none."""

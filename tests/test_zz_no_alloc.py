@@ -103,3 +103,19 @@ def test_noalloc_gemv_calls_on_two_streams_are_ordered():
     torch.cuda.synchronize()
     for i, (got, ref) in enumerate(zip(outs, want)):
         assert torch.equal(got, ref), f"call {i} on stream {i % 2} differs from the workspace GEMV"
+
+
+@pytest.mark.parametrize("m,n,k", [(2, 4096, 8960), (3, 2100, 14336), (5, 2100, 8960), (16, 2100, 5120), (4, 4096, 5120)])
+def test_noalloc_gemv_leaves_the_scratch_alone_where_it_can_do_without(m, n, k):
+    """Shapes that some kernel serves without partials: the no-alloc call is that kernel's, bit for bit the workspace
+    entry point without a workspace, so such calls share nothing over streams and captured graphs."""
+    print(f"no-alloc GEMV without scratch: M={m} N={n} K={k}", flush=True)
+    packed, qs, x, t, b = _problem(m, n, k, 16, 760)
+    w = _descriptor(packed, qs)
+    want = torch.empty((m, n), device="cuda", dtype=torch.bfloat16)
+    _lib.check(_lib.load().molt_nf4_gemv(x.data_ptr(), k, m, C.byref(w), t.data_ptr(), 16, b.data_ptr(), 16, 2.0,
+                                         want.data_ptr(), n, None, 0, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(_run(True, packed, qs, x, t, b, 2.0), want)
+    wo = oracle_weight(packed, qs).dequant_bf16().astype(np.float64)
+    ref = bf16_values(x) @ wo.T + 2.0 * (bf16_values(t) @ bf16_values(b).T)
+    assert_close_fro(np_f32(want), ref, what="no-alloc GEMV vs oracle")
