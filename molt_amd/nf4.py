@@ -21,6 +21,7 @@ from dataclasses import dataclass
 from typing import Any
 
 import torch
+from torch.utils._python_dispatch import _get_current_dispatch_mode
 
 from . import ops
 from .errors import CapabilityError
@@ -68,16 +69,27 @@ def dynamic_map(signed: bool = True, max_exponent_bits: int = 7, total_bits: int
 
 # The two code tables on each device, made once: building the dynamic map takes
 # some 80 us of host work and each upload waits for the device. Every weight
-# gets a copy of its own.
+# gets a copy of its own. Only plain eager code shares them: under a dispatch
+# mode (fake tensors among them), a functorch transform or torch.compile the
+# tables are that call's, or what the mode made of them would stay behind for
+# every later call.
 _TABLES: dict = {}
 
 
+def _upload(dev: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
+    return NF4_CODEBOOK.to(dev), dynamic_map().to(dev)
+
+
 def _tables(dev: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
+    if torch.compiler.is_compiling() or _get_current_dispatch_mode() is not None or \
+            torch._C._functorch.peek_interpreter_stack() is not None:
+        return _upload(dev)
     if dev.index is None:
         dev = torch.device(dev.type, torch.cuda.current_device())
     got = _TABLES.get(dev)
     if got is None:
-        got = _TABLES[dev] = (NF4_CODEBOOK.to(dev), dynamic_map().to(dev))
+        with torch.inference_mode(False):
+            got = _TABLES[dev] = _upload(dev)
     return got
 
 
@@ -149,14 +161,15 @@ def quantize_4bit(A: torch.Tensor, blocksize: int = 64, compress_statistics: boo
     if A.device.type != "cuda":
         raise CapabilityError("NF4 quantization requires a CUDA tensor on a ROCm GPU")
     dev = A.device
-    cb = _tables(dev)[0].clone() if code is None else code.to(dev, torch.float32)
+    tables = _tables(dev) if code is None or compress_statistics else None
+    cb = tables[0].clone() if code is None else code.to(dev, torch.float32)
     packed, absmax = ops.direct.nf4_quantize(A, blocksize, nibble_order, cb)
     n = A.numel()
     packed = packed[: (n + 1) // 2].reshape(-1, 1)
     dtype = A.dtype if A.dtype in (torch.bfloat16, torch.float16, torch.float32) else torch.bfloat16
     if not compress_statistics:
         return packed, QuantState(absmax, A.shape, cb, blocksize, "nf4", dtype, None, None, nibble_order)
-    code2 = _tables(dev)[1].clone()
+    code2 = tables[1].clone()
     q, absmax2, offset = ops.direct.nf4_double_quantize(absmax, code2, 256)
     state2 = QuantState(absmax2, (absmax2.numel(),), code2, 256, "dynamic", torch.float32)
     qs = QuantState(q, A.shape, cb, blocksize, "nf4", dtype, offset, state2, nibble_order)
