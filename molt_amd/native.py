@@ -251,10 +251,7 @@ def stacked_backward(dy: Tensor, x: Tensor, t: Tensor, packed, qs, wt: Tensor, a
     d = dy.device
     dx, da = _empty(d, _BF16, m, k), _empty(d, _F32, lr, k)
     dbs = [_empty(d, _F32, rw, r) for rw in rows]
-    key = ("molt_stacked_backward_workspace", m, tuple(rows), k, r, lr, _lib.tuning_generation)
-    size = ops._WS.get(key)
-    if size is None:
-        size = ops._WS[key] = int(_lib.load().molt_stacked_backward_workspace(m, n, (C.c_int64 * n)(*rows), k, r, lr))
+    size = ops._workspace("molt_stacked_backward_workspace", m, n, tuple(rows), k, r, lr)
     buf = _empty(d, _U8, size)
     pdb = (C.c_void_p * n)(*[b.data_ptr() for b in dbs])
     ops._call("molt_stacked_backward", dy.data_ptr(), x.data_ptr(), t.data_ptr(), m, n, ws, wt.data_ptr(),

@@ -129,13 +129,15 @@ def _f32(t: Tensor) -> Tensor:
 _WS: dict = {}
 
 
-def _workspace(query: str, *args: int) -> int:
+def _workspace(query: str, *args) -> int:
+    """``args``: numbers, or a tuple of them where the query takes an int64 array."""
     key = (query, args, _lib.tuning_generation)
     n = _WS.get(key)
     if n is None:
         if len(_WS) > 4096:
             _WS.clear()
-        n = _WS[key] = int(getattr(_lib.load(), query)(*args))
+        n = _WS[key] = int(getattr(_lib.load(), query)(*((C.c_int64 * len(a))(*a) if isinstance(a, tuple) else a
+                                                         for a in args)))
     return n
 
 

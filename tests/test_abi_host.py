@@ -231,6 +231,21 @@ def test_gemv_workspace_is_asked_only_where_k_is_split():
                                         (5, 4096, 5120), (16, 1536, 8960)))
 
 
+def test_kept_workspace_sizes_are_bounded_and_take_arrays():
+    """Every size that the host keeps goes through one bounded table, the stacked backward's (whose key holds the rows
+    of each projection) included; native.py adds to it by no other way."""
+    import ctypes
+    import inspect
+
+    from molt_amd import native, ops
+
+    rows = (1536, 256, 256)
+    got = [ops._workspace("molt_stacked_backward_workspace", m, 3, rows, 1536, 16, 64) for m in range(1, 5000)]
+    want = _lib.load().molt_stacked_backward_workspace(4096, 3, (ctypes.c_int64 * 3)(*rows), 1536, 16, 64)
+    assert got[4095] == want > 0 and len(ops._WS) <= 4097
+    assert "_WS" not in inspect.getsource(native)
+
+
 def test_split_k_workspace_queries_need_no_gpu():
     """The split plan: a long contraction with few 256 x 256 output tiles gets
     fp32 partials for S splits; a problem that fills the GPU gets none."""
