@@ -2077,7 +2077,7 @@ MOLT_DEV void contract(const Operands& o, int sbeg, int send, bool lora, const i
   for (int c = 0; c < 4; ++c) {
     xoff[c] = (uint32_t)((xrow[c] * o.ldx + kofs[c]) * 2);
     woff[c] = (uint32_t)((wrow[c] * o.ldw + kofs[c]) * 2);
-    // T's chunks past a short lr re-read the row's own columns: they meet zero adapter rows
+    // T's chunks past a short lr re-read the row's own columns; drop_t clears them
     toff[c] = (uint32_t)((xrow[c] * o.ldt + kofs[c] % max(o.lr, 1)) * 2);
     loffs[c] = (uint32_t)((wrow[c] * o.ldl + kofs[c]) * 2);
   }
@@ -2127,7 +2127,14 @@ MOLT_DEV void contract(const Operands& o, int sbeg, int send, bool lora, const i
   load(x3, w3, 3);
   wait_vm<3 * kDma>();                               // step 0 landed
   step_barrier();
-  auto step = [&](int j, const uint16_t* xc, const uint16_t* wc, uint16_t* xn, uint16_t* wn_) {
+  // A LoRA step shorter than 64 ranks: T past them meets zero adapter rows, and an infinite T would make that a NaN, so
+  // each wave clears those chunks of what it loaded, once it has landed.
+  auto drop_t = [&](uint16_t* x) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (kofs[c] >= o.lr) *reinterpret_cast<u32x4_t*>(x + (wave * 4 + c) * 512 + 8 * lane) = u32x4_t{0u, 0u, 0u, 0u};
+  };
+  auto step = [&](int j, const uint16_t* xc, const uint16_t* wc, uint16_t* xn, uint16_t* wn_, uint16_t* x1st) {
     frags(wc, xc, 0, a[0], b[0]);
     mfmas(a[1], b[1]);
     load(xn, wn_, j + 4);                            // into the buffers read at step j - 1
@@ -2138,21 +2145,22 @@ MOLT_DEV void contract(const Operands& o, int sbeg, int send, bool lora, const i
       mfmas(a[kk & 1], b[kk & 1]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    wait_vm<3 * kDma>();                             // step j + 1 landed; j + 2 .. j + 4 may fly
+    wait_vm<3 * kDma>();                             // step j + 1 landed (X in x1st); j + 2 .. j + 4 may fly
+    if (o.lr < BK && j + 1 >= n_main) drop_t(x1st);
     step_barrier();
   };
   int j = 0;
   for (; j + 5 <= n_all; j += 5) {
-    step(j, x0, w0, x4, w4);
-    step(j + 1, x1, w1, x0, w0);
-    step(j + 2, x2, w2, x1, w1);
-    step(j + 3, x3, w3, x2, w2);
-    step(j + 4, x4, w4, x3, w3);
+    step(j, x0, w0, x4, w4, x1);
+    step(j + 1, x1, w1, x0, w0, x2);
+    step(j + 2, x2, w2, x1, w1, x3);
+    step(j + 3, x3, w3, x2, w2, x4);
+    step(j + 4, x4, w4, x3, w3, x0);
   }
-  if (j < n_all) step(j, x0, w0, x4, w4);
-  if (j + 1 < n_all) step(j + 1, x1, w1, x0, w0);
-  if (j + 2 < n_all) step(j + 2, x2, w2, x1, w1);
-  if (j + 3 < n_all) step(j + 3, x3, w3, x2, w2);
+  if (j < n_all) step(j, x0, w0, x4, w4, x1);
+  if (j + 1 < n_all) step(j + 1, x1, w1, x0, w0, x2);
+  if (j + 2 < n_all) step(j + 2, x2, w2, x1, w1, x3);
+  if (j + 3 < n_all) step(j + 3, x3, w3, x2, w2, x4);
   mfmas(a[1], b[1]);
   wait_vm<0>();                                      // the repeated loads land before the workgroup ends
 }
