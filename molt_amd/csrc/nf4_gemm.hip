@@ -2485,6 +2485,8 @@ bool mid_wanted(const MidPlan& mid, const GemmPlan& plan, bool staged_big, int w
   const double stage = 4.5 + (double)weights * (double)rows * (double)cols * 2.5 / (backward ? 4e6 : 4.5e6);
   return 1.05 * (mid.cost + stage) < fused;
 }
+// Rows of a DMA operand through 32-bit buffer offsets.
+bool below_2g(int64_t rows, int64_t ld, int64_t cols) { return ((rows - 1) * ld + cols) * 2 < 0x7fffffffll; }
 size_t mid_stage_bytes(int weights, int64_t rows, int64_t cols, int64_t lora_rows, int64_t lr) {
   return weights * (stage_one(rows, cols) + (lr > 0 ? stage_one(lora_rows, ring_cols(lr)) : 0));
 }
@@ -2621,8 +2623,9 @@ extern "C" int molt_nf4_lora_forward_impl(const uint16_t* x, int64_t ldx, int64_
   const int nw = pair ? 2 : 1;
   const size_t msb = mid_stage_bytes(nw, p.N, p.K, p.N, lr);
   MidPlan mp;
-  const bool mid = al && mid_forward(plan, M, p.N, p.K, nw, lr, mp) && (lr == 0 || t_dma) &&
-                   ((M - 1) * ldx + p.K) * 2 < 0x7fffffffll && workspace && aligned(workspace, 256) &&
+  const bool mid = al && mid_forward(plan, M, p.N, p.K, nw, lr, mp) && below_2g(M, ldx, p.K) &&
+                   (lr == 0 || (t_dma && below_2g(M, ldt, lr) && below_2g(p.N, ring_cols(lr), ring_cols(lr)))) &&
+                   workspace && aligned(workspace, 256) &&
                    workspace_bytes >= msb + split_bytes(mp.S, M, p.N);
   if (mid) {
     const int lrc = lr > 0 ? (int)ring_cols(lr) : 0;
@@ -2893,10 +2896,11 @@ extern "C" int molt_nf4_lora_backward_impl(const uint16_t* dy0, const uint16_t* 
                  (long long)p.Nw, (long long)p.Kw);
   const size_t msb = mid_stage_bytes(nseg, p.Nw, p.Kw, p.Kw, r);
   MidPlan mp;
-  const bool u_dma = r == 0 || (aligned(u0, 16) && (nseg == 1 || aligned(u1, 16)) && ldu % 8 == 0);
+  const bool u_dma = r == 0 || (aligned(u0, 16) && (nseg == 1 || aligned(u1, 16)) && ldu % 8 == 0 &&
+                                below_2g(M, ldu, r) && below_2g(p.Kw, ring_cols(r), ring_cols(r)));
   const bool mid = al && mid_backward(plan, M, p.Nw, p.Kw, nseg, swiglu, r, mp) && u_dma && !use_wt &&
                    aligned(w0->packed, 4) && (nseg == 1 || aligned(w1->packed, 4)) &&
-                   ((M - 1) * lddy + p.Nw) * 2 < 0x7fffffffll && workspace && aligned(workspace, 256) &&
+                   below_2g(M, lddy, p.Nw) && workspace && aligned(workspace, 256) &&
                    workspace_bytes >= msb + split_bytes(mp.S, M, p.Kw);
   const int64_t np = (p.Nw + 63) / 64 * 64;
   MidPlan pp;

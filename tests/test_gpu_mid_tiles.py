@@ -49,3 +49,18 @@ def test_infinite_low_rank_value_stays_infinite(r):
     bad = ops.nf4_lora_backward_input(dy, *args, u, a, 1.0)
     keep = [i for i in range(m) if i != 3]
     assert torch.equal(bad[keep], dx[keep]) and torch.equal(bad[3].float(), a[0].sign() * float("-inf"))
+
+
+def test_low_rank_rows_far_apart():
+    """U rows whose stride puts the last one past 4 GiB: past the reach of the DMA's 32-bit offsets, so the call takes
+    the kernel that addresses them in 64 bits."""
+    m, n, k, r, ld = 70, 192, 320, 16, 32 * 1024 * 1024 + 8
+    (p0, s0, qs, w0), (p1, s1, _, w1) = _weight(n, k, 80), _weight(n, k, 81)
+    u = torch.empty((m - 1) * ld + 2 * r, device="cuda", dtype=torch.bfloat16).as_strided((m, 2 * r), (ld, 1))
+    u.copy_(seeded((m, 2 * r), 82))
+    dy0, dy1 = seeded((m, n), 83), seeded((m, n), 84)
+    a0, a1 = uniform((r, k), 85, 1.0 / np.sqrt(k)), uniform((r, k), 86, 1.0 / np.sqrt(k))
+    dx = ops.nf4_lora_backward_input_pair(dy0, dy1, p0, s0, p1, s1, qs.code, n, k, 1, u[:, :r], u[:, r:], a0, a1)
+    uu = bf16_values(u)
+    ref = bf16_values(dy0) @ w0 + bf16_values(dy1) @ w1 + uu[:, :r] @ bf16_values(a0) + uu[:, r:] @ bf16_values(a1)
+    assert_close_fro(np_f32(dx), ref, what="dX")
