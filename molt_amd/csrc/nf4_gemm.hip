@@ -2029,8 +2029,9 @@ struct Stager {
 // reads and MFMAs only, and the 160 KB of LDS hold a ring of five steps of both
 // operands, so a step's data is requested four steps before its use. Four waves
 // of 64 x 64; the last sub-step's MFMAs run under the next step's first reads.
-// The contraction runs in the fused kernels' order over the same split ranges,
-// so every output is bitwise theirs.
+// The products and their order along the contraction are the fused kernels'; the
+// ranges it is split into are mid_plan's own, so an output is bitwise theirs only
+// where those coincide, and elsewhere a sum of other fp32 partial sums.
 // ======================================================================
 namespace mid {
 
