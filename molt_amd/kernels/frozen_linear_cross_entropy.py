@@ -61,10 +61,12 @@ triton_frozen_loss_supported = fused_frozen_loss_supported
 
 def _hidden_grad(dlogits: torch.Tensor, weight: torch.Tensor, out: torch.Tensor) -> None:
     """``out = dlogits . weight``, the hidden gradient of one chunk: the split
-    HIP GEMM where it applies, else (and for the stand-in tensors of a tracing
-    pass) the library's."""
-    if ops._plain((dlogits, weight, out)) and weight.shape[0] == dlogits.shape[1] and out.dtype in (torch.bfloat16, torch.float32) and \
-            out.is_contiguous() and out.data_ptr() % 16 == 0 and ops.head_grad_applies(dlogits, weight):
+    HIP GEMM where it applies, else (and under torch.compile and for the
+    stand-in tensors of a tracing pass, which have no addresses to look at) the
+    library's."""
+    if not torch.compiler.is_compiling() and ops._plain((dlogits, weight, out)) \
+            and weight.shape[0] == dlogits.shape[1] and out.dtype in (torch.bfloat16, torch.float32) \
+            and out.is_contiguous() and out.data_ptr() % 16 == 0 and ops.head_grad_applies(dlogits, weight):
         ops.direct.head_grad(dlogits, weight, out)
     else:
         out.copy_(dlogits @ weight)

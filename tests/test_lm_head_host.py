@@ -39,3 +39,17 @@ def test_validation_errors():
         frozen_linear_cross_entropy(torch.randn(4, 16), w, t, 0)
     with pytest.raises(ValueError, match="Unknown backend"):
         exact_partitioned_linear_cross_entropy(torch.randn(4, 16), w, t, 2, backend="cuda")
+
+
+def test_hidden_gradient_of_a_chunk_traces():
+    """Under torch.compile the chunk's gradient is the library product, traced in one graph: nothing asks a traced
+    tensor for its address."""
+    from molt_amd.kernels.frozen_linear_cross_entropy import _hidden_grad
+
+    def grad(dlogits, weight, out):
+        _hidden_grad(dlogits, weight, out)
+        return out
+
+    d, w = torch.randn(2, 4096).bfloat16(), torch.randn(4096, 16).bfloat16()
+    got = torch.compile(grad, backend="eager", fullgraph=True)(d, w, torch.empty(2, 16, dtype=torch.bfloat16))
+    assert torch.equal(got, d @ w)
