@@ -15,6 +15,17 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 #define MOLT_DEV __device__ __forceinline__
 
 // ---------------------------------------------------------------------------
+// Waits until at most N of this wave's vector-memory operations (loads, stores,
+// DMA into LDS) are outstanding; the other counters are untouched. gfx9 splits
+// vmcnt over bits 3:0 and 15:14.
+// ---------------------------------------------------------------------------
+template <int N>
+MOLT_DEV void wait_vm() {
+  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+
+// ---------------------------------------------------------------------------
 // Vector-memory order. A partial vmcnt wait names operations by their place in
 // issue order: "at most N outstanding" means the N youngest. The compiler knows
 // which registers a load fills, but not that LDS filled by DMA is read after a

@@ -894,12 +894,6 @@ MOLT_DEV void gl_read4(const float* at, float (&u)[4]) {
                : "=&v"(u[0]), "=&v"(u[1]), "=&v"(u[2]), "=&v"(u[3]) : "v"(gl_addr(at)) : "memory");
 }
 
-template <int N>
-MOLT_DEV void gl_wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
-
 // slice_blocks: blocks of a K slice; wpg = ceil(slice_blocks / GL_BW) waves to a
 // group; gpr groups side by side; rounds = rounds of this grid.
 template <int SM, int LV, bool ONE>
@@ -985,7 +979,7 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
       loads_in_order();                      // round 0's wait counts every load of round 1 as younger
       if constexpr (!ONE) gl_load(b1, s1, p, wr, br, grp(1), blk, nb, lane, nr);
       __builtin_amdgcn_sched_barrier(0);
-      gl_wait_vm<(ONE ? 1 : 2) * GlRound<SM, LV>::kLoads>();
+      wait_vm<(ONE ? 1 : 2) * GlRound<SM, LV>::kLoads>();
       if constexpr (LV == 2) pack_t();
       asm volatile("" ::"v"(c2), "v"(tf) : "memory");      // older loads, landed: said here, where they can still be counted
 #pragma unroll
@@ -1001,7 +995,7 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
       __builtin_amdgcn_sched_barrier(0);
       gl_load(b0, s0, p, wr, br, grp(0), blk, nb, lane, nr);
       __builtin_amdgcn_sched_barrier(0);
-      gl_wait_vm<GlRound<SM, LV>::kLoads>();
+      wait_vm<GlRound<SM, LV>::kLoads>();
       if constexpr (LV == 2) pack_t();
       asm volatile("" ::"v"(c2), "v"(tf) : "memory");
       const uint8_t* at[GL_BW] = {s1, s2, xs, xs + GL_SLOT};
@@ -1082,7 +1076,7 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
   auto round = [&](int j, GlRound<SM, LV>& cur, const uint8_t* slot, GlRound<SM, LV>& nxt, uint8_t* into) {
     if constexpr (!ONE) gl_load(nxt, into, p, wr, br, grp(j + 2), blk, nb, lane, nr);
     __builtin_amdgcn_sched_barrier(0);
-    gl_wait_vm<kFly>();
+    wait_vm<kFly>();
     asm volatile("" ::: "memory");
     const f32x4_t acc = gl_compute(cur, slot, p, sm, lb, xf, tf, grp(j), blk, nb, nr, lane);
     reduce(j, &acc);
@@ -1095,7 +1089,7 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
     round(j, b2, s2, b1, s1);
     if (++j == rounds) break;
   }
-  gl_wait_vm<0>();                           // the repeated rounds land before the workgroup ends
+  wait_vm<0>();                           // the repeated rounds land before the workgroup ends
 }
 
 // Y[m, n] = bf16(sum over K slices of the fp32 partials), slices in order.

@@ -119,7 +119,7 @@ __global__ __launch_bounds__(NT) void head_grad_kernel(const HeadGradParams p) {
     d_load(db0, 0);
     loads_in_order();
     w_load(wb1, 1);
-    wait_vm_at_most<kStageDma>();
+    wait_vm<kStageDma>();
     step_barrier();
     auto step = [&](int j, const uint16_t* wc, const uint16_t* dc, uint16_t* w2, uint16_t* dnx) {
       load_frags_nn(wc, dc, ao, bo, 0, a[0], bf[0]);
@@ -134,11 +134,11 @@ __global__ __launch_bounds__(NT) void head_grad_kernel(const HeadGradParams p) {
         mfma_set(a[kk & 1], bf[kk & 1], acc);
         __builtin_amdgcn_sched_barrier(0);
       }
-      wait_vm_at_most<kStageDma>();                  // D(j + 1), W(j + 1) landed; W(j + 2) may fly
+      wait_vm<kStageDma>();                  // D(j + 1), W(j + 1) landed; W(j + 2) may fly
       step_barrier();
     };
     ring_steps(n, step, wb0, wb1, wb2, db0, db1);
-    wait_vm0();
+    wait_vm<0>();
     __syncthreads();
     mfma_set(a[1], bf[1], acc);
   }

@@ -301,14 +301,11 @@ MOLT_DEV void pj_dma16(__amdgpu_buffer_rsrc_t r, uint16_t* dst, uint32_t off, ui
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (pj_lds_t)dst, 16, off, soff, 0, 0);
 }
 
-// Wait until at most N vector-memory ops are outstanding (vmcnt N, other
-// counters untouched), with compiler barriers so no LDS read moves above the
-// wait. gfx9 splits vmcnt over bits 3:0 and 15:14.
+// wait_vm with compiler barriers, so that no LDS read moves above the wait.
 template <int N>
 MOLT_DEV void pj_wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
   asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+  wait_vm<N>();
   asm volatile("" ::: "memory");
 }
 

@@ -1175,7 +1175,7 @@ __global__ __launch_bounds__(NT) void fwd_kernel(const FwdParams p) {
     w_src(wb0, 0);
     loads_in_order();
     x_src(xb1, 1);
-    wait_vm_at_most<kStageDma>();                    // X(0), W(0) landed; X(1) may fly
+    wait_vm<kStageDma>();                    // X(0), W(0) landed; X(1) may fly
     step_barrier();
     // deq(W)^T for the input gradient: main step s of column tile tn is
     // written by the row block tm = s % nt_m, so each step's tile is written
@@ -1204,17 +1204,17 @@ __global__ __launch_bounds__(NT) void fwd_kernel(const FwdParams p) {
         mfma_set(a[kk & 1], b[kk & 1], acc);
         __builtin_amdgcn_sched_barrier(0);
       }
-      wait_vm_at_most<kStageDma>();                  // W(j + 1), X(j + 1) landed; X(j + 2) may fly
+      wait_vm<kStageDma>();                  // W(j + 1), X(j + 1) landed; X(j + 2) may fly
       step_barrier();
     };
     ring_steps(n_all, step, xb0, xb1, xb2, wb0, wb1);
-    wait_vm0();                                      // the last step's X(j + 2), never read
+    wait_vm<0>();                                      // the last step's X(j + 2), never read
     __syncthreads();
   } else {
     WBytes r0, r1;
     x_load(xb0, (int64_t)sbeg * BK);
     w_load(r0, (int64_t)sbeg * BK);
-    wait_vm0();
+    wait_vm<0>();
     __syncthreads();  // table, X(sbeg)
     {
       float2 c[4];
@@ -1222,7 +1222,7 @@ __global__ __launch_bounds__(NT) void fwd_kernel(const FwdParams p) {
       for (int d = 0; d < 4; ++d) { w_lookup(r0, tabc, d, c); w_finish(c, r0.sc, wb0, wR, wh, d); }
     }
     w_load(r0, min((int64_t)(sbeg + 1) * BK, klast));
-    wait_vm0();
+    wait_vm<0>();
     __syncthreads();
 
     auto step = [&](int s, const WBytes& cw, WBytes& nw, const uint16_t* xc, const uint16_t* wc, uint16_t* xn,
@@ -1246,7 +1246,7 @@ __global__ __launch_bounds__(NT) void fwd_kernel(const FwdParams p) {
         __builtin_amdgcn_sched_barrier(0);
       }
       w_finish(c, cw.sc, wnx, wR, wh, 3);
-      wait_vm_at_most<WBytes::kLoads>();            // X(s + 1) landed; only W(s + 2)'s loads may fly
+      wait_vm<WBytes::kLoads>();            // X(s + 1) landed; only W(s + 2)'s loads may fly
       step_barrier();
     };
     // W(s + 1) sits in r0 during even steps and in r1 during odd ones; the LDS buffers alternate likewise.
@@ -1662,7 +1662,7 @@ __global__ __launch_bounds__(NT) void bwd_kernel(const BwdParams p) {
     w_dma(wb0, sbeg);
     loads_in_order();
     x_load(xb1, sbeg + 1);
-    wait_vm_at_most<kStageDma>();                    // dY(sbeg), W(sbeg) landed; dY(sbeg + 1) may fly
+    wait_vm<kStageDma>();                    // dY(sbeg), W(sbeg) landed; dY(sbeg + 1) may fly
     step_barrier();
     auto step = [&](int s, const uint16_t* xc, const uint16_t* wc, uint16_t* x2, uint16_t* wnx) {
       load_frags(wc, xc, fo, 0, a[0], b[0]);
@@ -1677,7 +1677,7 @@ __global__ __launch_bounds__(NT) void bwd_kernel(const BwdParams p) {
         mfma_set(a[kk & 1], b[kk & 1], acc);
         __builtin_amdgcn_sched_barrier(0);
       }
-      wait_vm_at_most<kStageDma>();                  // W(s + 1), dY(s + 1) landed; dY(s + 2) may fly
+      wait_vm<kStageDma>();                  // W(s + 1), dY(s + 1) landed; dY(s + 2) may fly
       step_barrier();
     };
     // buffers of step s: dY s % 3, W s % 2, so the pattern repeats every 6 steps
@@ -1699,17 +1699,17 @@ __global__ __launch_bounds__(NT) void bwd_kernel(const BwdParams p) {
       step(s, xb2, wb0, xb1, wb1);
       step(s + 1, xb0, wb1, xb2, wb0);
     }
-    wait_vm0();                                      // the last step's dY(s + 2), never read
+    wait_vm<0>();                                      // the last step's dY(s + 2), never read
     __syncthreads();
   } else {
     WPatch r0, r1;
     x_load(xb0, sbeg);
     w_load(r0, sbeg);
-    wait_vm0();
+    wait_vm<0>();
     __syncthreads();  // table, X(sbeg)
     wp_commit(r0, tabc, wb0, cg, rg);
     w_load(r0, sbeg + 1);
-    wait_vm0();
+    wait_vm<0>();
     __syncthreads();
 
     // Dequant of W(s+1) across the sub-steps: column pairs (0,1), (4,5) then
@@ -1749,7 +1749,7 @@ __global__ __launch_bounds__(NT) void bwd_kernel(const BwdParams p) {
       wp_finish(c, cw.sc, c4, c5);
       wp_swap_write(c0, c4, wnx, cg, rg, 2);
       wp_swap_write(c1, c5, wnx, cg, rg, 3);
-      wait_vm_at_most<WPatch::kLoads>();            // dY(s + 1) landed; only W(s + 2)'s loads may fly
+      wait_vm<WPatch::kLoads>();            // dY(s + 1) landed; only W(s + 2)'s loads may fly
       step_barrier();
     };
     for (int s = sbeg; s < send; s += 2) {
@@ -2046,13 +2046,6 @@ using big::step_barrier;
 constexpr int MBUF = 128 * 64;      // bf16 elements of one operand buffer (16 KB)
 constexpr int kDma = 8;             // DMA instructions per wave and step, both operands
 static_assert(BM == 128 && BN == 128 && NT == 256, "four waves fill 16 KB per operand with 4 DMA instructions each");
-
-// vmcnt(N) for N up to 63 (the immediate's high bits are 15:14), other counters untouched.
-template <int N>
-MOLT_DEV void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
 
 // Operands of the contraction: nseg main segments of ks steps, then nseg LoRA
 // segments of ls steps. X and T are indexed by segment; W and its adapter rows

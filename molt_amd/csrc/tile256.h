@@ -89,15 +89,6 @@ MOLT_DEV uint32_t buf_load4(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t sof
 MOLT_DEV void buf_load_lds16(__amdgpu_buffer_rsrc_t r, void* dst, uint32_t off, uint32_t soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 16, off, soff, 0, 0);
 }
-// vmcnt(N) with the other counters untouched: wait until at most N of this
-// wave's vector-memory operations (loads, buffer-to-LDS DMA) are outstanding.
-template <int N>
-MOLT_DEV void wait_vm_at_most() {
-  static_assert(N >= 0 && N < 16, "vmcnt immediate is 4 bits here");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | N);
-}
-MOLT_DEV void wait_vm0() { wait_vm_at_most<0>(); }
-
 // Workgroup barrier without __syncthreads()'s release fence: the fence makes
 // the compiler drain every outstanding vector-memory op, including register
 // loads of packed weight bytes that are only used a step later. The caller
