@@ -456,3 +456,12 @@ def test_gemv_three_and_four_tokens_over_three_pieces(m, n, k, r):
         t, b = seeded((m, r), 802), seeded((n, r), 803, std=0.01, dtype=torch.float32)
         ref = ref + s * (bf16_values(t) @ bf16_values(b).T)
     assert_close_fro(np_f32(_gemv(x, packed, qs, t, b, s)), ref, what="Y")
+
+
+def test_gemv_with_the_adapter_passes_opcheck():
+    n, k, r = 64, 128, 8
+    packed, qs = molt_amd.quantize_4bit(seeded((n, k), 900, std=0.02, dtype=torch.float32))
+    s2 = qs.state2
+    torch.library.opcheck(ops.nf4_lora_gemv, (
+        seeded((3, k), 901), packed.reshape(-1), None, qs.absmax, s2.absmax, s2.code, float(qs.offset), 256, qs.code, n,
+        k, 1, uniform((r, k), 902, 0.1), seeded((n, r), 903, std=0.01, dtype=torch.float32), 2.0))

@@ -268,3 +268,9 @@ def test_head_grad_refuses_what_it_does_not_take():
         ops.head_grad(d, w, out[:3])
     with pytest.raises(ValueError):
         ops.head_grad(d, w.repeat(2, 1), out)
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_head_gradient_passes_opcheck(out_dtype):
+    d, w = (torch.randn(*s, device="cuda").bfloat16() for s in ((5, 4096), (4096, 64)))
+    torch.library.opcheck(ops.head_grad, (d, w, torch.empty(5, 64, device="cuda", dtype=out_dtype)))
