@@ -296,7 +296,7 @@ void nf4_gemv_kernel(const GemvParams p, float* part) {
 
 
 // ---------------------------------------------------------------------------
-// Streaming dot-product variant for M <= 4 (decode). Each wave walks rows of W
+// Streaming dot-product variant for few tokens (decode; see dot_serves). Each wave walks rows of W
 // in rounds: round j covers RW rows at j * (grid waves * RW) + (this wave's
 // index) * RW, so every round of the grid reads a contiguous band of W. A
 // lane reads 16 contiguous packed bytes (32 elements, half a block) of each
@@ -672,6 +672,8 @@ void nf4_gemv_dot_kernel(const GemvParams p, int rounds) {
 //   M = 5    7.06 6.57 6.78  13.96 13.75 14.04  17.44 16.49 16.85  10.52 7.93 7.62   14.00 10.64 10.40  7.38 6.70 6.04
 //   M = 8    7.79 7.13 6.82  14.33 14.28 14.31  18.28 17.28 17.03  11.16 8.34 7.72   15.24 11.18 10.53  7.79 7.35 6.07
 //   M = 16   9.11 8.46 7.44  16.13 15.53 15.06  19.90 18.48 17.91  12.64 9.44 8.32   18.04 12.21 11.04  9.01 8.64 6.50
+// Since then (groups by gl_plan, B by buffer loads), one run on a box whose large shapes are 6% slower: M = 5 6.6,
+// 14.7, 16.4, 7.5, 10.5, 5.1; M = 8 6.6, 14.6, 16.6, 7.5, 10.6, 5.1; M = 16 7.1, 15.7, 17.4, 7.6, 11.1, 5.4.
 // Ranks that are no multiple of 8 take B by the same two loads a round; one load and address per rank cost, M = 5:
 // 14336 x 4096 at rank 4 / 5 / 12 21.8 / 21.2 / 22.2 -> 14.2 / 15.4 / 13.8, 8960 x 1600 16.9 / 16.0 / 17.6 -> 9.9 /
 // 10.4 / 9.7 (weights through registers, ranks by fours: 14.2 / 16.1 / 13.7, 10.7 / 10.7 / 10.9).
@@ -925,7 +927,9 @@ void nf4_gemv_lds_kernel(const GemvParams p, int slice_blocks, int wpg, int gpr,
   if constexpr (LV != 0) {
     // Ranks past r, and waves without ranks of this slice, load from outside the
     // buffer: zeros, no traffic (T gathered by all waves cost 0.4 us a token) and
-    // no branch or select that would wait for the load here.
+    // no branch or select that would wait for the load here. (In the forms of one
+    // round the M <= 8 side below still begins with a wait for it: the two sides
+    // share registers.)
     const __amdgpu_buffer_rsrc_t tr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(p.t), (short)0, (int)(((int64_t)(p.M - 1) * p.ldt + p.r) * 2), 0x00020000);
     const int j = jc + 8 * g;
@@ -1228,9 +1232,11 @@ static bool gemv_needs_workspace(int64_t M, int64_t K) {
 // Kilobyte pieces of a row, and whether the dot kernel serves a call by its
 // sizes (with 16-byte aligned codes). M = 1, 2 always. Up to 8 tokens over at
 // most 2048 rows and K <= 4096 (eight X rows of at most two pieces fit in LDS
-// beside the code table): eight tokens per lookup, where the MFMA kernel leaves
+// beside the code table): eight tokens per lookup, where the MFMA kernel left
 // most CUs idle (M = 8: 2048^2 5.4 / 6.8 us, 1536^2 5.3 / 5.6; 1024 x 4096 6.5 /
-// 6.9; M = 4: 1536^2 4.0 / 5.3, 2048 x 8192 7.8 / 9.0). M = 3, 4 with three
+// 6.9. With its groups side by side only where they pay that kernel takes 5.1, 4.6
+// and 6.0 there, from five tokens on: this line has not been moved yet. M = 4:
+// 1536^2 4.1 / 4.5, 2048 x 8192 7.9 / 8.9, 1536 x 8960 7.7 / 10.3). M = 3, 4 with three
 // pieces over at most 4096 rows, two rounds of the grid, where the MFMA kernel
 // runs two slices, two or more rounds and their sum (4096 x 4160 8.5 / 11.1 us, 2112
 // x 5120 8.1 / 9.5, 4096 x 6144 8.8 / 11.1; but 4608 x 5120 13.0 / 11.3, and with
