@@ -211,6 +211,10 @@ constexpr int QZ_BUCKETS = 129;
 constexpr int QZ_UNITS = 2;
 // Workgroups per CU: each builds the table once and strides over the blocks.
 constexpr int QZ_GRID_PER_CU = 8;
+// Blocks per CU from which the table pays: below, its 2 us of bisection outweigh the scan, a wave per block. Scan
+// and table from bf16 on the MI355X (256 CUs): 64 blocks 2.8 and 4.6 us, 6144 3.9 and 4.9, 9216 4.7 and 4.9, 10,240
+// 4.9 and 4.9, 11,264 5.1 and 4.9, 16,384 6.3 and 5.0; the same line from fp32.
+constexpr int QZ_MIN_BLOCKS_PER_CU = 40;
 
 template <int IN_BF16, bool ALIGNED>
 __global__ __launch_bounds__(CODEC_NT) void quantize64_kernel(const void* __restrict__ x, int64_t n, int order,
@@ -317,7 +321,8 @@ __global__ __launch_bounds__(CODEC_NT) void quantize64_kernel(const void* __rest
   }
 }
 
-// Any other block size (and codes that are not 4-byte aligned): a wave per block, a pair of elements per lane.
+// Any other block size, few blocks of 64 and codes that are not 4-byte aligned: a wave per block, one element (blocks
+// of 64) or a pair of elements per lane.
 template <int IN_BF16>
 __global__ __launch_bounds__(CODEC_NT) void quantize_kernel(const void* __restrict__ x, int64_t n,
                                                             int block, int order,
@@ -335,6 +340,31 @@ __global__ __launch_bounds__(CODEC_NT) void quantize_kernel(const void* __restri
     if (IN_BF16) return bf16_to_f32(reinterpret_cast<const uint16_t*>(x)[i]);
     return reinterpret_cast<const float*>(x)[i];
   };
+  if (block == 64) {
+    // each element loaded once, QB blocks per pass with every load issued before the first is used; the odd lane's
+    // code joins its even neighbour's by a lane shift and the even lanes store the bytes
+    constexpr int QB = 4;
+    for (int64_t b0 = (int64_t)blockIdx.x * (CODEC_NT / 64) + (threadIdx.x >> 6); b0 < nblocks; b0 += QB * waves) {
+      float v[QB];
+#pragma unroll
+      for (int k = 0; k < QB; ++k) {
+        const int64_t b = b0 + k * waves;
+        v[k] = b < nblocks ? load(b * 64 + lane) : 0.0f;
+      }
+#pragma unroll
+      for (int k = 0; k < QB; ++k) {
+        const int64_t b = b0 + k * waves;
+        if (b >= nblocks) break;   // uniform across the wave
+        const float am = fmaxf(wave_max(fmaxf(0.0f, fabsf(v[k]))), 1.17549435e-38f);
+        if (lane == 0) absmax[b] = am;
+        const uint32_t bi = nearest16(cb, v[k] / am);
+        const uint32_t odd = (uint32_t)__shfl_down((int)bi, 1, 64);
+        if ((lane & 1) == 0)
+          packed[b * 32 + (lane >> 1)] = (uint8_t)(order ? ((bi << 4) | odd) : (bi | (odd << 4)));
+      }
+    }
+    return;
+  }
   for (int64_t b = (int64_t)blockIdx.x * (CODEC_NT / 64) + (threadIdx.x >> 6); b < nblocks; b += waves) {
     const int64_t base = b * block;
     float m = 0.0f;
@@ -546,7 +576,8 @@ extern "C" int molt_nf4_quantize(const void* x, int32_t x_dtype, int64_t n, int3
   MOLT_REQUIRE(nibble_order == 0 || nibble_order == 1, MOLT_EINVAL, "%s: bad nibble order", who);
   const int64_t nblocks = ceil_div64(n, block_size);
   hipStream_t st = (hipStream_t)stream;
-  if (block_size == 64 && aligned(packed, 4)) {   // the codes are stored 4 bytes at a time
+  if (block_size == 64 && nblocks >= QZ_MIN_BLOCKS_PER_CU * device_cus() &&
+      aligned(packed, 4)) {                       // the codes are stored 4 bytes at a time
     const int64_t g64 = ceil_div64(nblocks, 8 * QZ_UNITS * (CODEC_NT / 64));
     const dim3 grid64((unsigned)std::min<int64_t>(g64, QZ_GRID_PER_CU * device_cus()));
     const bool al = aligned(x, 16), b16 = x_dtype == MOLT_DTYPE_BF16;

@@ -47,7 +47,7 @@ def test_quantize_special_values(block):
 
 def test_quantize_block64_more_blocks_than_one_pass():
     """135,168 blocks of 64: more than one pass of the block-64 path's grid
-    (8192 workgroups x 4 waves x 4 blocks), the second pass partial."""
+    (2048 workgroups x 4 waves x 2 units of 8 blocks), the second pass partial."""
     shape = (4096, 2112)
     print(f"quantize block64 multi-pass shape={shape}", flush=True)
     x = seeded(shape, 7, std=0.02, dtype=torch.bfloat16)
@@ -130,8 +130,8 @@ _TABLES = {
 @pytest.mark.parametrize("n", [2, 64, 65, 64 * 7 + 6, 64 * 8, 64 * 9 + 62, 64 * 8 * 4 * 3 + 34])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_quantize_block64_against_the_scan(n, dtype, table):
-    """Block 64 (8 lanes to a block, one threshold per bucket) at the edges of its units, for tables it looks up and
-    tables it scans, from aligned and unaligned inputs: every code and absmax as the definition's scan."""
+    """Few blocks of 64 (a wave to a block) at the edges of a wave's and a pass's blocks, for each kind of table, from
+    aligned and unaligned inputs: every code and absmax as the definition's scan."""
     print(f"quantize block64 n={n} dtype={dtype} table={table}", flush=True)
     code = _TABLES[table]
     x = seeded((n + 1,), 900 + n, std=0.02, dtype=dtype)
@@ -160,6 +160,50 @@ def test_quantize_block64_at_the_thresholds_and_out_of_range_blocks():
         idx, am = O.quantize_blocks(x, 64)
     assert np.array_equal(np_f32(absmax).view(np.uint32), am.view(np.uint32))
     assert np.array_equal(packed.cpu().numpy(), O.pack_nibbles(idx, 0))
+
+
+def _table_blocks():
+    """Blocks of 64 from which the quantiser looks its codes up (below, it scans them): 40 per CU."""
+    return 40 * torch.cuda.get_device_properties(0).multi_processor_count
+
+
+@pytest.mark.parametrize("table", list(_TABLES))
+@pytest.mark.parametrize("extra", [-64, -63, 0, 64 * 8 * 4 * 3 + 34])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_quantize_block64_around_the_table_line(extra, dtype, table):
+    """Just below, at and above the number of blocks where the quantiser goes from the scan to the threshold table,
+    with whole and ragged last blocks, aligned and unaligned inputs and every kind of table."""
+    n = _table_blocks() * 64 + extra
+    print(f"quantize block64 n={n} dtype={dtype} table={table}", flush=True)
+    code = _TABLES[table]
+    x = seeded((n + 1,), 950 + extra % 7, std=0.02, dtype=dtype)
+    for src in (x[:n].clone(), x[1:]):
+        packed, absmax = ops.nf4_quantize(src, 64, 1, torch.from_numpy(code).cuda())
+        idx, am = O.quantize_blocks(np_f32(src), 64, code)
+        assert np.array_equal(np_f32(absmax).view(np.uint32), am.view(np.uint32))
+        assert np.array_equal(packed.cpu().numpy(), O.pack_nibbles(idx, 1))
+
+
+def test_quantize_block64_thresholds_through_the_table():
+    """The floats around every midpoint, and blocks out of the reciprocal's range, in a weight large enough for the
+    threshold table; eight equal blocks in a row, so that whole waves of blocks are in range and take it."""
+    mids = (O.NF4_CODE[:-1].astype(np.float64) + O.NF4_CODE[1:]) / 2
+    rows = []
+    for am in (1.0, 0.0213, 3.7e-3, 1.999999, 2.0 ** -59, 2.0 ** 59, 2.0 ** -61, 2.0 ** 61, 1e-38, 3e38):
+        for step in range(-4, 5):
+            near = (mids * am).astype(np.float32)
+            for _ in range(abs(step)):
+                near = np.nextafter(near, np.float32(np.inf if step > 0 else -np.inf))
+            rows.append(np.concatenate([near, -near, [np.float32(am)], np.zeros(33, np.float32)]))
+    rows += [np.zeros(64), np.full(64, 1e-45), np.r_[np.inf, np.zeros(62), 1.0]]
+    x = np.repeat(np.stack(rows).astype(np.float32), 8, axis=0)
+    times = -(-_table_blocks() // len(x))
+    packed, absmax = ops.nf4_quantize(torch.from_numpy(np.tile(x, (times, 1))).cuda(), 64, 0,
+                                      molt_amd.NF4_CODEBOOK.cuda())
+    with np.errstate(invalid="ignore"):
+        idx, am = O.quantize_blocks(x, 64)
+    assert np.array_equal(np_f32(absmax).view(np.uint32), np.tile(am.reshape(-1), times).view(np.uint32))
+    assert np.array_equal(packed.cpu().numpy().reshape(times, -1), np.tile(O.pack_nibbles(idx, 0).reshape(1, -1), (times, 1)))
 
 
 @pytest.mark.parametrize("table", ["dynamic", "ties", "unsorted"])
